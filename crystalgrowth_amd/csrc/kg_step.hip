@@ -1406,7 +1406,7 @@ __device__ __forceinline__ void multi_tile(const StepArgs<R> &a, int x0, int y0,
 #pragma unroll
     for (int w = 0; w < NT / 64; ++w)
         fl &= sm.W[w];
-    const bool flat = fl != 0;
+    bool flat = fl != 0;
     const R pc = (fl & 1) ? (R)0 : (R)1;
 
     // the LDS cell a thread's cell takes its neighbours from: itself, or for a
@@ -1451,6 +1451,7 @@ __device__ __forceinline__ void multi_tile(const StepArgs<R> &a, int x0, int y0,
             __syncthreads();
         }
         R pn[S::TQ], tn[S::TQ];
+        bool finite = true;  // of a flat step's T
 #pragma unroll
         for (int t = 0; t < S::TQ; ++t) {
             if (ring[t] > oh)
@@ -1462,6 +1463,7 @@ __device__ __forceinline__ void multi_tile(const StepArgs<R> &a, int x0, int y0,
             if (flat) {
                 pn[t] = pc;
                 tn[t] = Tc + lapT * a.dt + a.K * (pc - pc);
+                finite = finite && isfinite(tn[t]);
                 continue;
             }
             const R *pz = &sm.P[(lr + 1) * PW + lc], *pm = pz - PW, *pp = pz + PW;
@@ -1508,8 +1510,24 @@ __device__ __forceinline__ void multi_tile(const StepArgs<R> &a, int x0, int y0,
                 a.theta[o] = th[t];
             }
         }
-        if (s < K)
+        if (s < K) {
+            // T that overflowed in a flat step reaches phi in the next one, as
+            // it does between single steps, which look at T anew: the full
+            // path from here on
+            if (flat) {
+                const bool w = __ballot(!finite) == 0;
+                if ((tid & 63) == 0)
+                    sm.W[tid >> 6] = w ? 1 : 0;
+            }
             __syncthreads();
+            if (flat) {
+                int all = 1;
+#pragma unroll
+                for (int w = 0; w < NT / 64; ++w)
+                    all &= sm.W[w];
+                flat = all != 0;
+            }
+        }
     }
 }
 
