@@ -1173,6 +1173,13 @@ __global__ __launch_bounds__(S::NT) void k_step_small(StepArgs<R> a)
                 all0 = all1 = 0;
         }
     }
+    // a kept angle that is not finite (the bound behind wide_angles would show
+    // it) makes phi NaN whatever phi is
+    if (a.wide_angles)
+#pragma unroll
+        for (int t = 0; t < S::TQ; ++t)
+            if (!isfinite(th[t]))
+                all0 = all1 = 0;
     {
         const bool w0 = __ballot(all0) == __ballot(1), w1 = __ballot(all1) == __ballot(1);
         if ((tid & 63) == 0)
@@ -1404,6 +1411,11 @@ __device__ __forceinline__ void multi_tile(const StepArgs<R> &a, int x0, int y0,
                 all0 = all1 = 0;
         }
     }
+    if (a.wide_angles)  // (as in k_step_small)
+#pragma unroll
+        for (int t = 0; t < S::TQ; ++t)
+            if (!isfinite(th[t]))
+                all0 = all1 = 0;
     {
         const bool w0 = __ballot(all0) == __ballot(1), w1 = __ballot(all1) == __ballot(1);
         if ((tid & 63) == 0)
