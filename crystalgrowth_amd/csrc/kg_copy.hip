@@ -13,20 +13,13 @@
 //
 // Pinned buffers are shared by all handles: at most STAGES of STAGE_MAX bytes,
 // each held by one call at a time, all freed with the last handle.  A call that
-// finds none, and memory that the runtime knows (pinned, managed or device),
-// copies directly.
-#include <sys/mman.h>
-#include <unistd.h>
-
-#include <cerrno>
+// finds none, memory that the runtime knows (pinned, managed or device), and
+// memory that the processor may not write copy directly.
 #include <cstring>
 #include <mutex>
 
 #include "kg_host.h"
-
-#ifndef MADV_POPULATE_WRITE
-#define MADV_POPULATE_WRITE 23
-#endif
+#include "kg_stage.h"
 
 namespace kg {
 
@@ -112,16 +105,6 @@ bool pageable(const void *p)
     return a.type == hipMemoryTypeUnregistered;
 }
 
-// Pages of [p, p + n) present and writable; false where the kernel says that
-// they cannot be (where it cannot tell, the copy faults them in).
-bool populate(void *p, size_t n)
-{
-    static const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
-    const uintptr_t lo = (uintptr_t)p & ~(page - 1);
-    return madvise((void *)lo, (uintptr_t)p + n - lo, MADV_POPULATE_WRITE) == 0 ||
-           (errno != EFAULT && errno != ENOMEM);
-}
-
 hipError_t copy_direct(hipStream_t s, const HostPiece *pieces, int count)
 {
     for (int k = 0; k < count; ++k)
@@ -169,7 +152,7 @@ hipError_t copy_staged(hipStream_t s, const HostPiece *pieces, int count, char *
         if (hipError_t e = hipStreamSynchronize(s))
             return e;
         if (!ok)
-            return copy_direct(s, pieces, count);  // the runtime's to refuse
+            return copy_direct(s, pieces, count);  // the runtime's to copy or refuse
         if (hipError_t e = fill(h ^ 1))
             return e;
         for (int k = 0; k < np[h]; ++k)
