@@ -11,12 +11,12 @@
 // 16 MB 1650 / 1270 and 940 / 630, 64 MB 6590 / 4940.  (The other direction
 // stays with the runtime: 37 GB/s, and 28 GB/s this way.)
 //
-// Pinned buffers are shared by all handles: at most STAGES of STAGE_MAX bytes,
-// each held by one call at a time, all freed with the last handle.  A call that
-// finds none, memory that the runtime knows (pinned, managed or device), and
-// memory that the processor may not write copy directly.
+// Pinned buffers are shared by all handles: at most STAGES of STAGE_MAX bytes
+// (kg_stage.h), each held by one call at a time, all freed with the last
+// handle.  A call that finds none, memory that the runtime knows (pinned,
+// managed or device), and memory that the processor may not write copy
+// directly.
 #include <cstring>
-#include <mutex>
 
 #include "kg_host.h"
 #include "kg_stage.h"
@@ -24,21 +24,6 @@
 namespace kg {
 
 namespace {
-
-constexpr int STAGES = 8;
-constexpr size_t STAGE_MIN = (size_t)512 << 10, STAGE_MAX = (size_t)4 << 20;
-// The first buffer costs some 13 us, a small copy through it saves 8: it is
-// made for a copy of this size, or the fourth.
-constexpr size_t WORTH_A_STAGE = (size_t)256 << 10;
-constexpr int WORTH_COPIES = 4;
-
-std::mutex g_mutex;
-struct Stage {
-    char *p;
-    size_t cap;
-    bool used;
-} g_stages[STAGES];
-int g_handles = 0, g_copies = 0;
 
 // Allocating is harmless to a capture that is under way elsewhere in this
 // process, but the runtime refuses it in the default capture mode.
@@ -48,51 +33,20 @@ struct RelaxedCapture {
     ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// A free buffer, of twice `bytes` if that is within the limits; -1: none.
-int take_stage(size_t bytes)
-{
-    size_t cap = STAGE_MIN;
-    while (cap < 2 * bytes && cap < STAGE_MAX)
-        cap *= 2;
-    std::lock_guard<std::mutex> lock(g_mutex);
-    int at = -1;
-    for (int k = 0; k < STAGES; ++k) {
-        const Stage &g = g_stages[k];
-        if (g.used)
-            continue;
-        if (g.cap >= cap) {
-            at = k;
-            break;
-        }
-        if (at < 0 || g.cap > g_stages[at].cap)
-            at = k;  // the largest too small (or empty) one grows
-    }
-    if (at < 0)
-        return -1;
-    Stage &g = g_stages[at];
-    if (g.cap < cap) {
-        if (g.cap == 0 && bytes < WORTH_A_STAGE && ++g_copies < WORTH_COPIES)
-            return -1;
+StagePool g_stages(
+    [](size_t cap) -> void * {
         const RelaxedCapture relaxed;
-        if (g.p)
-            (void)hipHostFree(g.p);
-        g = Stage{nullptr, 0, false};
         void *p = nullptr;
         if (hipHostMalloc(&p, cap, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
-            return -1;
+            return nullptr;
         }
-        g = Stage{static_cast<char *>(p), cap, false};
-    }
-    g.used = true;
-    return at;
-}
-
-void give_stage(int at)
-{
-    std::lock_guard<std::mutex> lock(g_mutex);
-    g_stages[at].used = false;
-}
+        return p;
+    },
+    [](void *p) {
+        const RelaxedCapture relaxed;
+        (void)hipHostFree(p);
+    });
 
 // Memory that the runtime does not know: pageable.
 bool pageable(const void *p)
@@ -171,34 +125,18 @@ hipError_t copy_to_host(hipStream_t s, const HostPiece *pieces, int count)
         total += (pieces[k].bytes + 255) / 256 * 256;
         staged = staged && pageable(pieces[k].host);
     }
-    const int at = staged ? take_stage(total) : -1;
+    const int at = staged ? g_stages.take(total) : -1;
     if (at < 0)
         return copy_direct(s, pieces, count);
-    const hipError_t e = copy_staged(s, pieces, count, g_stages[at].p, g_stages[at].cap / 2);
+    const hipError_t e =
+        copy_staged(s, pieces, count, g_stages.buffer(at), g_stages.capacity(at) / 2);
     if (e != hipSuccess)
         (void)hipStreamSynchronize(s);  // nothing writes to the buffer any more
-    give_stage(at);
+    g_stages.give(at);
     return e;
 }
 
-void stages_retain()
-{
-    std::lock_guard<std::mutex> lock(g_mutex);
-    ++g_handles;
-}
-
-void stages_release()
-{
-    std::lock_guard<std::mutex> lock(g_mutex);
-    if (--g_handles > 0)
-        return;
-    const RelaxedCapture relaxed;
-    for (Stage &g : g_stages) {
-        if (g.p)
-            (void)hipHostFree(g.p);
-        g = Stage{nullptr, 0, false};
-    }
-    g_copies = 0;
-}
+void stages_retain() { g_stages.retain(); }
+void stages_release() { g_stages.release(); }
 
 }  // namespace kg
