@@ -250,10 +250,9 @@ int init_fields(kg_solver_s &h, const std::vector<int> &cxy, double r2)
     std::vector<kg::DiskEntry> d(cxy.size() / 2);
     for (size_t k = 0; k < d.size(); ++k)
         d[k] = kg::DiskEntry{0, h.nx, h.ny, cxy[2 * k], cxy[2 * k + 1]};
-    R *phi = static_cast<R *>(h.phi[0]);
-    KG_HIP(kg::launch_zero<R>(phi, static_cast<R *>(h.T[0]), static_cast<R *>(h.theta), h.cells(),
-                              h.stream));
-    if (int rc = kg::draw_disks<R>(phi, d, r2, h.disks, h.disks_cap, h.stream))
+    if (int rc = kg::reset_fields<R>(static_cast<R *>(h.phi[0]), static_cast<R *>(h.T[0]),
+                                     static_cast<R *>(h.theta), h.cells(), d, r2, h.partials,
+                                     h.disks, h.disks_cap, h.stream))
         return rc;
     KG_HIP(hipStreamSynchronize(h.stream));
     h.steps = 0;

@@ -611,19 +611,18 @@ int step_impl(kg_batch_s &b, int nsteps)
     return launch_steps(b, nsteps);
 }
 
-// Members lo .. hi - 1: all fields 0, phi = 1 on the disks (of those members)
-// of squared radius r2.  A member's fields are padded to 256 bytes, so the
-// members are one range of every buffer.
+// Members lo .. hi - 1: all fields 0, phi = 1 on the disks (of those members,
+// offsets from the first one's fields) of squared radius r2.  A member's fields
+// are padded to 256 bytes, so the members are one range of every buffer.
 template <typename R>
 int init_members(kg_batch_s &b, int lo, int hi, const std::vector<kg::DiskEntry> &disks, double r2)
 {
     const int c = b.cur();
     invalidate_status(b);
-    const size_t end = hi < b.count ? b.off[hi] : b.total;
-    R *phi = static_cast<R *>(b.phi[c]);
-    KG_HIP(kg::launch_zero<R>(phi + b.off[lo], static_cast<R *>(b.T[c]) + b.off[lo],
-                              static_cast<R *>(b.theta) + b.off[lo], end - b.off[lo], b.stream));
-    if (int rc = kg::draw_disks<R>(phi, disks, r2, b.disks, b.disks_cap, b.stream))
+    const size_t at = b.off[lo], end = hi < b.count ? b.off[hi] : b.total;
+    if (int rc = kg::reset_fields<R>(static_cast<R *>(b.phi[c]) + at, static_cast<R *>(b.T[c]) + at,
+                                     static_cast<R *>(b.theta) + at, end - at, disks, r2, b.partials,
+                                     b.disks, b.disks_cap, b.stream))
         return rc;
     KG_HIP(hipStreamSynchronize(b.stream));
     return KG_OK;
@@ -640,7 +639,7 @@ int init_disk(kg_batch_s &b, int lo, int hi, int cx, int cy, double r2)
 {
     std::vector<kg::DiskEntry> d;
     for (int m = lo; m < hi; ++m)
-        d.push_back(kg::DiskEntry{b.off[m], b.nx[m], b.ny[m], cx < 0 ? b.nx[m] / 2 : cx,
+        d.push_back(kg::DiskEntry{b.off[m] - b.off[lo], b.nx[m], b.ny[m], cx < 0 ? b.nx[m] / 2 : cx,
                                   cx < 0 ? b.ny[m] / 2 : cy});
     return init_members(b, lo, hi, d, r2);
 }
@@ -851,7 +850,8 @@ int kg_batch_reset_seeds(kg_batch b, int member, int count, double r, int margin
     for (int m = lo; m < hi; ++m) {
         kg::seed_centres(b->nx[m], b->ny[m], count, margin, seed, d.data());
         for (int k = 0; k < count; ++k)
-            disks.push_back(kg::DiskEntry{b->off[m], b->nx[m], b->ny[m], d[2 * k], d[2 * k + 1]});
+            disks.push_back(kg::DiskEntry{b->off[m] - b->off[from], b->nx[m], b->ny[m], d[2 * k],
+                                          d[2 * k + 1]});
         if (m + 1 < hi && disks.size() < kg::DISK_CHUNK)
             continue;
         if (int rc = init_members(*b, from, m + 1, disks, r * r))

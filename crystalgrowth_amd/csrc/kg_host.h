@@ -48,7 +48,7 @@ struct kg_solver_s {
     void *temps = nullptr;  // 6 fields, two-pass kernel only
     double *partials = nullptr;
     kg::ReduceOut *red = nullptr;
-    kg::DiskEntry *disks = nullptr;  // nuclei of a reset
+    kg::DiskEntry *disks = nullptr;  // nuclei of a reset that are too many for partials
     size_t disks_cap = 0;
     void *image = nullptr;  // colours of the last ramp, up to IMAGE_KEEP bytes
     size_t image_cap = 0;
@@ -110,7 +110,7 @@ struct kg_batch_s {
     uint32_t *step_base = nullptr;
     double *partials = nullptr;
     kg::ReduceOut *red = nullptr;
-    kg::DiskEntry *disks = nullptr;  // nuclei of a reset
+    kg::DiskEntry *disks = nullptr;  // nuclei of a reset that are too many for partials
     size_t disks_cap = 0;
     uint64_t steps = 0;        // steps since the last reset of all members
     uint64_t base_host = 0;    // value of *step_base
@@ -249,15 +249,33 @@ inline int max_abs(const void *v, size_t n, int precision, double *partials, hip
     return KG_OK;
 }
 
-// phi = 1 on the disks (entries uploaded through the device buffer `dev` of
-// `cap` entries, grown as needed up to DISK_CHUNK; longer lists go in turns).
+// n elements of each field 0 but for phi = 1 on the disks.  A few disks of the
+// grid at phi travel with the launch; a list goes to the device in the reduction
+// scratch, or, if it is longer, in the buffer `dev` of `cap` entries, grown as
+// needed up to DISK_CHUNK (longer lists go in turns).
 constexpr size_t DISK_CHUNK = 65536;
 template <typename R>
-int draw_disks(R *phi, const std::vector<DiskEntry> &disks, double r2, DiskEntry *&dev, size_t &cap,
-               hipStream_t s)
+int reset_fields(R *phi, R *T, R *theta, size_t n, const std::vector<DiskEntry> &disks, double r2,
+                 double *scratch, DiskEntry *&dev, size_t &cap, hipStream_t s)
 {
+    FewDisks few{};
+    bool all = disks.size() <= (size_t)FewDisks::MAX;
+    for (const DiskEntry &d : disks) {
+        all = all && d.off == 0;
+        if (!all)
+            break;
+        few.cx[few.n] = d.cx;
+        few.cy[few.n++] = d.cy;
+    }
+    if (!all)
+        few.n = 0;
+    const int nx = disks.empty() ? 0 : disks[0].nx, ny = disks.empty() ? 0 : disks[0].ny;
+    KG_HIP(launch_reset<R>(phi, T, theta, n, nx, ny, few, r2, s));
+    if (all)
+        return KG_OK;
     const size_t want = disks.size() < DISK_CHUNK ? disks.size() : DISK_CHUNK;
-    if (want > cap) {
+    const bool fits = want * sizeof(DiskEntry) <= reduce_partials_size() * sizeof(double);
+    if (!fits && want > cap) {
         if (dev)
             KG_HIP(hipFree(dev));
         dev = nullptr;
@@ -265,11 +283,12 @@ int draw_disks(R *phi, const std::vector<DiskEntry> &disks, double r2, DiskEntry
         KG_HIP(hipMalloc(&dev, want * sizeof(DiskEntry)));
         cap = want;
     }
+    DiskEntry *list = fits ? reinterpret_cast<DiskEntry *>(scratch) : dev;
     for (size_t at = 0; at < disks.size(); at += want) {
-        const size_t n = disks.size() - at < want ? disks.size() - at : want;
-        KG_HIP(hipMemcpyAsync(dev, disks.data() + at, n * sizeof(DiskEntry), hipMemcpyHostToDevice,
+        const size_t m = disks.size() - at < want ? disks.size() - at : want;
+        KG_HIP(hipMemcpyAsync(list, disks.data() + at, m * sizeof(DiskEntry), hipMemcpyHostToDevice,
                               s));
-        KG_HIP(launch_disks<R>(phi, dev, (int)n, r2, s));
+        KG_HIP(launch_disks<R>(phi, list, (int)m, r2, s));
     }
     return KG_OK;
 }

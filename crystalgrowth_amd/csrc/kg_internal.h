@@ -147,15 +147,24 @@ hipError_t launch_step_two_pass(const StepArgs<R> &a, const PassTemps<R> &t, hip
 // Bytes to allocate for a field of `bytes`: whole 16-byte words, so that
 // fields can be cleared with 16-byte stores.
 constexpr size_t padded_bytes(size_t bytes) { return (bytes + 15) / 16 * 16; }
-// All fields zero (n elements each, allocated with padded_bytes).
-template <typename R>
-hipError_t launch_zero(R *phi, R *T, R *theta, size_t n, hipStream_t s);
-// phi = 1 on disks of squared radius r2 (the reference's 5-cell plus is the
-// disk with r2 = 1); off: element offset of the grid in phi.
+// A disk of phi = 1 (the reference's 5-cell plus is the disk with r2 = 1); off:
+// element offset of its grid in phi.
 struct DiskEntry {
     size_t off;
     int nx, ny, cx, cy;
 };
+// Centres of disks that travel with a launch.
+struct FewDisks {
+    static constexpr int MAX = 8;
+    int n;
+    int cx[MAX], cy[MAX];
+};
+// All fields zero (n elements each, allocated with padded_bytes) but for phi on
+// the disks of squared radius r2 in the nx x ny grid at phi.
+template <typename R>
+hipError_t launch_reset(R *phi, R *T, R *theta, size_t n, int nx, int ny, const FewDisks &disks,
+                        double r2, hipStream_t s);
+// phi = 1 on `count` disks of squared radius r2 (a list in device memory).
 template <typename R>
 hipError_t launch_disks(R *phi, const DiskEntry *disks, int count, double r2, hipStream_t s);
 

@@ -2126,17 +2126,48 @@ __global__ __launch_bounds__(256) void k_pass2(StepArgs<R> a, PassTemps<R> t)
 }
 
 // ---- initial states -------------------------------------------------------
-// All fields 0, then phi = 1 on the disks: two kernels, each bound by its
-// stores.  One kernel asking every cell about every disk took 592 us on a
-// 4096 x 4096 FP32 grid with 200 disks (600 FP64 operations per cell); these
-// two take 27 + 3.5 us (192 MiB of zeros and 200 boxes of 11 x 11 cells).
-__global__ __launch_bounds__(256) void k_zero3(uint4 *a, uint4 *b, uint4 *c, size_t n)
+// All fields 0, and phi = 1 on the few disks of an nx x ny grid that travel with
+// the launch: a reset to one nucleus is one launch and nothing is uploaded for
+// it (512 x 512: 18 -> 12 us).  More disks are drawn by k_disks: one kernel asking
+// every cell about every disk took 592 us on a 4096 x 4096 FP32 grid with 200
+// disks (600 FP64 operations per cell); these two take 27 + 3.5 us (192 MiB of
+// zeros and 200 boxes of 11 x 11 cells).  q: 16-byte words per field, one per
+// thread in turn (4096 x 4096 FP64: 76 us; four per thread, a quarter of the field
+// apart, 92); k: a disk lies within cy +- k.
+template <typename R>
+__global__ __launch_bounds__(256) void k_reset(R *phi, R *T, R *theta, size_t q, int nx, int ny,
+                                               FewDisks d, double r2, long long k)
 {
+    constexpr int V = 16 / sizeof(R);
     const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        a[i] = z;
-        b[i] = z;
-        c[i] = z;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < q; i += (size_t)gridDim.x * 256) {
+        R v[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            v[e] = (R)0;
+        for (int m = 0; m < d.n; ++m) {
+            // the cells of the rows that the disk touches
+            const long long y0 = d.cy[m] - k > 0 ? d.cy[m] - k : 0;
+            const long long y1 = d.cy[m] + k < ny - 1 ? d.cy[m] + k : ny - 1;
+            const size_t lo = y0 <= y1 ? (size_t)y0 * nx : 0;
+            const size_t hi = y0 <= y1 ? (size_t)(y1 + 1) * nx : 0;
+            if (i * V >= hi || i * V + V <= lo)
+                continue;
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                const size_t c = i * V + e;
+                const size_t j = c >> 32 ? c / nx : (uint32_t)c / (uint32_t)nx;
+                const double dj = (double)((long long)j - d.cy[m]);
+                const double di = (double)((long long)(c - j * nx) - d.cx[m]);
+                if (c >= lo && c < hi && di * di + dj * dj <= r2)
+                    v[e] = (R)1;
+            }
+        }
+        uint4 w;
+        __builtin_memcpy(&w, v, 16);
+        reinterpret_cast<uint4 *>(phi)[i] = w;
+        reinterpret_cast<uint4 *>(T)[i] = z;
+        reinterpret_cast<uint4 *>(theta)[i] = z;
     }
 }
 
@@ -2753,14 +2784,23 @@ hipError_t launch_step_two_pass(const StepArgs<R> &a, const PassTemps<R> &t, hip
     return hipGetLastError();
 }
 
+namespace {
+// Cells a disk of squared radius r2 reaches from its centre (at most 2^32)
+long long disk_reach(double r2)
+{
+    const double rad = ceil(sqrt(r2));
+    return rad < 4294967296.0 ? (long long)rad : 4294967296ll;
+}
+}  // namespace
+
 template <typename R>
-hipError_t launch_zero(R *phi, R *T, R *theta, size_t n, hipStream_t s)
+hipError_t launch_reset(R *phi, R *T, R *theta, size_t n, int nx, int ny, const FewDisks &disks,
+                        double r2, hipStream_t s)
 {
     // fields are 16-byte aligned and padded to 16 bytes (padded_bytes)
     const size_t q = (n * sizeof(R) + 15) / 16;
-    hipLaunchKernelGGL(k_zero3, dim3(grid_1d(q, 256 * 4)), dim3(256), 0, s,
-                       reinterpret_cast<uint4 *>(phi), reinterpret_cast<uint4 *>(T),
-                       reinterpret_cast<uint4 *>(theta), q);
+    hipLaunchKernelGGL((k_reset<R>), dim3(grid_1d(q, 256)), dim3(256), 0, s, phi, T, theta, q, nx,
+                       ny, disks, r2, disk_reach(r2));
     return hipGetLastError();
 }
 
@@ -2769,8 +2809,7 @@ hipError_t launch_disks(R *phi, const DiskEntry *disks, int count, double r2, hi
 {
     if (count <= 0)
         return hipSuccess;
-    const double rad = ceil(sqrt(r2));
-    const long long k = rad < 4294967296.0 ? (long long)rad : 4294967296ll;
+    const long long k = disk_reach(r2);
     // 8 box rows per block, and at most about 65536 blocks
     const long long rows = (2 * k + 8) / 8, most = std::max(1, 65536 / count);
     const dim3 grid(count, (unsigned)std::min(std::min(rows, most), 4096ll));
@@ -2904,7 +2943,8 @@ hipError_t launch_front_profile(const R *phi, int nx, int ny, double cx, double 
                                                     R *, uint32_t, hipStream_t);                 \
     template hipError_t launch_step_two_pass<R>(const StepArgs<R> &, const PassTemps<R> &,       \
                                                 hipStream_t);                                    \
-    template hipError_t launch_zero<R>(R *, R *, R *, size_t, hipStream_t);                      \
+    template hipError_t launch_reset<R>(R *, R *, R *, size_t, int, int, const FewDisks &,       \
+                                        double, hipStream_t);                                    \
     template hipError_t launch_disks<R>(R *, const DiskEntry *, int, double, hipStream_t);       \
     template hipError_t launch_reduce<R>(const R *, const R *, size_t, double, double *,         \
                                          ReduceOut *, hipStream_t);                              \
