@@ -745,7 +745,7 @@ int kg_set_fields(kg_handle h, const void *phi, const void *T, const void *theta
     h->theta_given = theta ? HUGE_VAL : 0.0;
     if (theta) {
         KG_HIP(hipMemcpyAsync(h->theta, theta, bytes, hipMemcpyHostToDevice, h->stream));
-        return kg::max_abs(h->theta, h->cells(), h->precision, h->partials, h->stream,
+        return kg::max_abs(theta, h->theta, h->cells(), h->precision, h->partials, h->stream,
                            &h->theta_given);  // waits for the stream
     }
     KG_HIP(hipMemsetAsync(h->theta, 0, bytes, h->stream));

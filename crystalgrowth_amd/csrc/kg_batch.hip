@@ -885,7 +885,7 @@ int kg_batch_set_fields(kg_batch b, int member, const void *phi, const void *T,
     // the member's angle bound decides its sin/cos path: refresh its table entry
     b->theta_given[member] = theta ? HUGE_VAL : 0.0;
     if (theta) {
-        if (int rc = kg::max_abs(b->field(b->theta, member), b->cells(member), b->precision,
+        if (int rc = kg::max_abs(theta, b->field(b->theta, member), b->cells(member), b->precision,
                                  b->partials, b->stream, &b->theta_given[member]))
             return rc;  // (it waits for the stream)
     } else {

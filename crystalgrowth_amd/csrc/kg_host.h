@@ -231,19 +231,35 @@ inline int wide_angles(const kg_params &p, double theta_given)
     return m <= 0.99e4 ? 0 : 1;
 }
 
-// Largest |v| of n device values of the given precision (NaN -> infinity),
-// through the reduction scratch `partials`; waits for the stream.  On the
-// host the same scan of a caller's array took 5.3 ms for 2048 x 2048 FP32
-// values; k_max_abs takes 11 us.
-inline int max_abs(const void *v, size_t n, int precision, double *partials, hipStream_t s,
-                   double *out)
+// Largest |v| of n values of the given precision (NaN -> infinity), which are at
+// `host` and, once the stream's copies have run, at `dev`; waits for the stream.
+// Few values are scanned on the host, 1.3 ns each (5.3 ms for 2048 x 2048): k_max_abs
+// and the copy of its partial maxima, through the reduction scratch `partials`,
+// take 14 us at least (and 25 us for 2048 x 2048 FP32 values).  kg_set_fields, us,
+// host / device: 96^2 cells FP32 33 / 46, FP64 34 / 48; 128^2 39 / 48, 42 / 53; 250^2
+// 109 / 62, 122 / 79.
+constexpr size_t HOST_SCAN = 24576;
+inline int max_abs(const void *host, const void *dev, size_t n, int precision, double *partials,
+                   hipStream_t s, double *out)
 {
+    double m = 0.0;
+    if (n <= HOST_SCAN) {
+        for (size_t i = 0; i < n; ++i) {
+            const double x = precision == KG_F64 ? static_cast<const double *>(host)[i]
+                                                 : (double)static_cast<const float *>(host)[i];
+            const double a = std::fabs(x);
+            if (!(a <= m))
+                m = a == a ? a : HUGE_VAL;
+        }
+        KG_HIP(hipStreamSynchronize(s));
+        *out = m;
+        return KG_OK;
+    }
     double part[MAX_ABS_BLOCKS];
     KG_HIP(precision == KG_F64
-               ? launch_max_abs<double>(static_cast<const double *>(v), n, partials, s)
-               : launch_max_abs<float>(static_cast<const float *>(v), n, partials, s));
+               ? launch_max_abs<double>(static_cast<const double *>(dev), n, partials, s)
+               : launch_max_abs<float>(static_cast<const float *>(dev), n, partials, s));
     KG_HIP(copy_to_host(s, part, partials, sizeof(part)));
-    double m = 0.0;
     for (double x : part)
         m = x > m ? x : m;
     *out = m;
