@@ -15,6 +15,8 @@
 namespace kg {
 
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+// (to a float's precision)
+__device__ __forceinline__ double fast_rcp(double x) { return __builtin_amdgcn_rcp(x); }
 
 // atan(q) for q in [0, 1]: q * A(q^2)
 __device__ __forceinline__ float atan_unit(float q)

@@ -1386,12 +1386,13 @@ __device__ __forceinline__ void multi_tile(const StepArgs<R> &a, int x0, int y0,
         sm.Z[0] = e0;
         sm.Z[1] = f0;
     }
-    // A flat tile steps T alone, so T must stay finite to the last step, as
-    // phi is NaN in the step after T is.  A step's 9-point sum is at most 24
-    // times the largest |T|, and T grows by a factor of 4 at most (dt / dx^2 <=
-    // 3 / 8).  (Asking T anew after each step: 250^2 FP32 2.3 -> 2.5 us a step.)
-    constexpr R GROWTH = (R)(24 << 2 * K);
-    const R limit = std::numeric_limits<R>::max() / (GROWTH * fmax((R)1, a.inv_3dx2));
+    // A flat tile steps T alone, so T must be finite before each of its steps, as
+    // phi is NaN in the step after T is.  A step's 9-point sum is at most 24 times
+    // the largest |T|, and T grows by a factor of 4 at most (dt / dx^2 <= 3 / 8).
+    // (Asking T anew after each step: 250^2 FP32 2.3 -> 2.5 us a step.)
+    constexpr R MOST = std::numeric_limits<R>::max() / (R)(48 << 2 * K);
+    const R limit = K == 1 ? std::numeric_limits<R>::infinity()
+                           : MOST * fast_rcp(fmax((R)1, a.inv_3dx2));
     int all0 = 1, all1 = 1;
 #pragma unroll
     for (int t = 0; t < S::TP; ++t) {
