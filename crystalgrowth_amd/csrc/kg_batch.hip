@@ -59,7 +59,7 @@ void free_batch(kg_batch_s *b)
     void *bufs[] = {b->phi[0], b->phi[1], b->T[0], b->T[1], b->theta, b->members,
                     b->tiles, b->step_base, b->partials, b->red, b->disks, b->stat,
                     b->chunks_dev, b->tiles_listed, b->dflags2, b->dcount, b->dperiods,
-                    b->multi_tiles, b->multi_off, b->theta_alt};
+                    b->multi_tiles, b->multi_off, b->theta_alt, b->members_plain};
     for (void *p : bufs)
         if (p)
             (void)hipFree(p);
@@ -478,6 +478,9 @@ int make_multi(kg_batch_s &b)
     // frees what was allocated)
     if (hipMalloc(&b.multi_tiles, dealt.size() * sizeof(int4)) != hipSuccess ||
         hipMalloc(&b.multi_off, b.off.size() * sizeof(size_t)) != hipSuccess ||
+        hipMalloc(&b.members_plain,
+                  b.count * (sizeof(kg::StepArgs<double>) + sizeof(kg::AdjMember<double>))) !=
+            hipSuccess ||
         hipMalloc(&b.theta_alt, b.total * b.esize()) != hipSuccess) {
         (void)hipGetLastError();
         return KG_OK;
@@ -490,25 +493,74 @@ int make_multi(kg_batch_s &b)
     return KG_OK;
 }
 
-// Pairs of launches of MULTI_STEPS steps: an odd number of steps moves phi
-// and T to the other buffer, as single steps would, and a pair leaves theta in
-// its own (the other modes' graphs and tables hold its address).
+// The batch's buffers for a step or launch that moves phi and T to the other
+// ones and theta from buffer k (0: theta, 1: theta_alt) to the other.
 template <typename R>
-int multi_pairs(kg_batch_s &b, int &n)
+kg::MultiIO<R> buffers(const kg_batch_s &b, int k)
+{
+    const int c = b.cur();
+    void *const th[2] = {b.theta, b.theta_alt};
+    return {static_cast<const R *>(b.phi[c]), static_cast<const R *>(b.T[c]),
+            static_cast<const R *>(th[k]), static_cast<R *>(b.phi[c ^ 1]),
+            static_cast<R *>(b.T[c ^ 1]), static_cast<R *>(th[k ^ 1])};
+}
+
+// Launches of MULTI_STEPS steps: an odd number of steps moves phi and T to the
+// other buffer, as single steps would.  theta has to end in its own buffer (the
+// other modes' graphs and tables hold its address), so they go in pairs; of the
+// steps left over, four or five take one more launch and a single step that
+// hands theta back.  The rest are 64 x 30 tiles without tile status, which these
+// launches do not keep: cleared for so few steps it cost more than it saved.  8
+// x 500^2 FP32 from one nucleus each, us per step in calls of 7 / 10 / 11 steps:
+// 9.8 / 9.7 / 9.8 in 64 x 30 tiles alone, 10.5 / 11.1 / 11.1 with the status
+// cleared for what is left over, 9.8 / 9.6 / 9.9 this way.
+template <typename R>
+int multi_steps(kg_batch_s &b, int n)
 {
     invalidate_status(b);
     const int steps = kg::multi_shape_steps(b.multi_shape);
-    while (n >= 2 * steps) {
+    for (; n >= 2 * steps; n -= 2 * steps)
         for (int k = 0; k < 2; ++k) {
-            const int c = b.cur();
-            void *th[2] = {b.theta, b.theta_alt};
-            const kg::MultiIO<R> io{static_cast<const R *>(b.phi[c]), static_cast<const R *>(b.T[c]),
-                                    static_cast<const R *>(th[k]), static_cast<R *>(b.phi[c ^ 1]),
-                                    static_cast<R *>(b.T[c ^ 1]), static_cast<R *>(th[k ^ 1])};
-            KG_HIP(kg::batch_multi<R>(b, io, (uint32_t)b.steps, 0));
+            KG_HIP(kg::batch_multi<R>(b, buffers<R>(b, k), (uint32_t)b.steps, 0));
             b.steps += (uint64_t)steps;
         }
-        n -= 2 * steps;
+    if (n == 0)
+        return KG_OK;
+    using Args = kg::StepArgs<R>;
+    using Member = kg::AdjMember<R>;
+    if (!b.plain_valid) {  // the members without tile status, alone and with their offsets
+        const size_t at = b.count * sizeof(Args);
+        // (what changes a member waits for the stream, so the last upload is over)
+        b.plain_host.resize(at + b.count * sizeof(Member));
+        const std::vector<Args> v = member_args<R>(b);
+        for (int m = 0; m < b.count; ++m) {
+            Member e{v[m], b.off[m]};
+            e.a.stat_in = nullptr;
+            e.a.stat_out = nullptr;
+            std::memcpy(&b.plain_host[m * sizeof(Args)], &e.a, sizeof(Args));
+            std::memcpy(&b.plain_host[at + m * sizeof(Member)], &e, sizeof(Member));
+        }
+        KG_HIP(hipMemcpyAsync(b.members_plain, b.plain_host.data(), b.plain_host.size(),
+                              hipMemcpyHostToDevice, b.stream));
+        b.plain_valid = true;
+    }
+    const Args *const plain = static_cast<const Args *>(b.members_plain);
+    if (n > steps) {
+        KG_HIP(kg::batch_multi<R>(b, buffers<R>(b, 0), (uint32_t)b.steps, 0));
+        b.steps += (uint64_t)steps;
+        const kg::MultiIO<R> io = buffers<R>(b, 1);
+        KG_HIP(kg::launch_step_batch_direct<R>(reinterpret_cast<const Member *>(plain + b.count),
+                                               b.tiles, b.ntiles, io.phi_in, io.T_in, io.theta_in,
+                                               io.phi_out, io.T_out, io.theta_out,
+                                               (uint32_t)b.steps, b.stream));
+        b.steps += 1;
+        n -= steps + 1;
+    }
+    for (; n > 0; --n) {
+        KG_HIP(kg::launch_step_batch<R>(plain, b.tiles, b.ntiles, b.step_base,
+                                        (uint32_t)(b.steps - b.base_host), boundary_mode(b),
+                                        b.stream, nullptr));
+        b.steps += 1;
     }
     return KG_OK;
 }
@@ -517,8 +569,7 @@ int launch_steps(kg_batch_s &b, int n)
 {
     if (b.multi_shape != 0 && b.mode == KG_BATCH_LAUNCH &&
         n >= 2 * kg::multi_shape_steps(b.multi_shape))
-        if (int rc = b.precision == KG_F64 ? multi_pairs<double>(b, n) : multi_pairs<float>(b, n))
-            return rc;
+        return b.precision == KG_F64 ? multi_steps<double>(b, n) : multi_steps<float>(b, n);
     if (n > 0)
         if (int rc = ensure_status(b))
             return rc;
@@ -781,6 +832,7 @@ int kg_batch_set_params(kg_batch b, int member, const kg_params *p)
     KG_HIP(hipStreamSynchronize(b->stream));
     const int bcm = boundary_mode(*b);
     b->params[member] = *p;
+    b->plain_valid = false;
     if (boundary_mode(*b) != bcm)
         drop_graph(b);  // it launches the step kernel compiled for the old boundary mix
     invalidate_status(*b);
@@ -884,6 +936,7 @@ int kg_batch_set_fields(kg_batch b, int member, const void *phi, const void *T,
         KG_HIP(hipMemsetAsync(b->field(b->theta, member), 0, bytes, b->stream));
     // the member's angle bound decides its sin/cos path: refresh its table entry
     b->theta_given[member] = theta ? HUGE_VAL : 0.0;
+    b->plain_valid = false;
     if (theta) {
         if (int rc = kg::max_abs(theta, b->field(b->theta, member), b->cells(member), b->precision,
                                  b->partials, b->stream, &b->theta_given[member]))

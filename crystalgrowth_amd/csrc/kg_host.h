@@ -127,11 +127,16 @@ struct kg_batch_s {
     bool stat_valid = false;
     std::vector<double> theta_given;  // per member, as kg_solver_s::theta_given
     // launches of several steps (shape 0: none; kg_step.hip, k_batch_multi):
-    // tile table, member offsets, and the other theta buffer (launch mode)
+    // tile table, member offsets, and the other theta buffer (launch mode); the
+    // member tables without tile status for the steps they leave over, and
+    // whether these hold the members' current parameters
     int multi_shape = 0, nmulti = 0;
     int4 *multi_tiles = nullptr;
     size_t *multi_off = nullptr;
     void *theta_alt = nullptr;
+    void *members_plain = nullptr;
+    std::vector<char> plain_host;  // source of its uploads
+    bool plain_valid = false;
     // chunk lists (launch mode, batches of at least SKIP_MIN_CHUNKS chunks;
     // kg_batch.hip, batch_skip_cycle): the chunks in the order the tile
     // table deals them (member, chunk column, chunk row), the pinned flags
