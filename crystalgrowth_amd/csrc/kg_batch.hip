@@ -1226,10 +1226,15 @@ int kg_batch_autotune(kg_batch b, int trial_steps, int *mode, int *graph_steps)
                           {KG_BATCH_GRAPH_LISTS, 8, 0, 0}, {KG_BATCH_GRAPH_LISTS, 32, 0, 0}};
     int shapes[16][2];
     const int nshapes = std::min(kg::batch_chunk_shapes(shapes, 16), 16);
+    // launches of several steps go by whole pairs, and in tiles of their own: one
+    // candidate, whatever the chunk shape
+    const int whole = b->multi_shape != 0 ? 2 * kg::multi_shape_steps(b->multi_shape) : 0;
     std::vector<Cand> cands;
+    if (whole)
+        cands.push_back({KG_BATCH_LAUNCH, 0, b->cw, b->ch});
     for (int k = 0; k < nshapes; ++k)
         for (const Cand &f : forms)
-            if (f.mode == KG_BATCH_LAUNCH || f.g <= trial_steps)
+            if (f.mode == KG_BATCH_LAUNCH ? !whole : f.g <= trial_steps)
                 cands.push_back({f.mode, f.g, shapes[k][0], shapes[k][1]});
     double best = 1e300;
     Cand pick = {b->mode, b->graph_steps, b->cw, b->ch};
@@ -1240,10 +1245,13 @@ int kg_batch_autotune(kg_batch b, int trial_steps, int *mode, int *graph_steps)
         if (rc == KG_OK)
             rc = kg_batch_set_mode(b, cd.mode, cd.g);
         double ms = 0.0;
+        const int pairs = cd.mode == KG_BATCH_LAUNCH ? whole : 0;
+        const int n = pairs ? (trial_steps + pairs - 1) / pairs * pairs : trial_steps;
         if (rc == KG_OK)
-            rc = kg_batch_step(b, cd.g > 0 ? cd.g : 2);  // warm up (capture, caches)
+            rc = kg_batch_step(b, cd.g > 0 ? cd.g : (pairs ? pairs : 2));  // warm up (capture, caches)
         if (rc == KG_OK)
-            rc = kg_batch_step_timed(b, trial_steps, &ms);
+            rc = kg_batch_step_timed(b, n, &ms);
+        ms *= (double)trial_steps / n;
         // restore the state before the next candidate
         b->steps = steps0;
         invalidate_status(*b);

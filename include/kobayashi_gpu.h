@@ -265,7 +265,8 @@ int kg_batch_get_chunk_shape(kg_batch b, int *chunk_w, int *chunk_h);
 /* Times trial_steps steps of each launch configuration (launch form and
  * chunk shape) on a copy of the current state and keeps the fastest (the
  * state is restored afterwards; kg_batch_get_chunk_shape reports the shape
- * it picked).  The chunk lists take effect within two liveness periods
+ * it picked).  KG_BATCH_LAUNCH of small batches, whose launches go by up to six
+ * steps whatever the chunk shape, is timed once, over whole launches.  The chunk lists take effect within two liveness periods
  * (14 steps) of the trial's start, so trials shorter than that time the
  * launch of every chunk. */
 int kg_batch_autotune(kg_batch b, int trial_steps, int *mode, int *graph_steps);

@@ -1,4 +1,5 @@
-"""Steps that whole pairs of launches of a small batch leave over (needs a GPU).
+"""Steps that whole pairs of launches of a small batch leave over, and the tuner's
+choice for such batches (needs a GPU).
 
 The left-over steps run without tile status, from a member table of their own:
 it follows changes of parameters, fields and angle bounds between calls, and
@@ -51,3 +52,20 @@ def test_left_over_steps_follow_the_members(kb, prec):
             else:
                 for c in (a, b):
                     c.reset_disk(m, -1, -1, 4.0)
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("trial", [2, 4, 16])
+def test_tuner_times_whole_launches(kb, trial, prec):
+    """Several steps a launch take a third of the time of one step a launch on
+    batches of this size, so launch mode wins however short the trial is."""
+    sizes = [(100, 100)] * 5
+    with kb.Batch(sizes, kb.default_params(noise_a=0.01), prec) as b:
+        b.reset_disk(-1, -1, -1, 6.0)
+        b.step(61)
+        before = [b.fields(m) for m in range(5)]
+        assert b.autotune(trial)[0] == "launch"
+        assert b.step_count == 61
+        for m in range(5):
+            for x, y in zip(before[m], b.fields(m)):
+                assert np.array_equal(x, y), m
