@@ -96,10 +96,18 @@ kg::StepArgs<R> make_args(const kg_solver_s &h)
 
 // Tile status is kept on grids of more than 2 Mi cells (the small tiles end
 // there at the latest), where the boundary allows it.  Below, its loads and
-// stores saved are worth less than the round trip to the status words: FP32
-// 1472 x 1424, us per step with / without, 16.2 / 13.9 with one nucleus per
-// 60000 cells, 7.7 / 8.1 with one in all; 1800 x 1800 20.8 / 17.9 and 9.0 /
-// 10.5.
+// stores saved are worth less than the round trip to the status words.  us per
+// step with / without, steps 0 .. 100 and 1500 .. 1800, one nucleus per 60000
+// cells and one in all:
+//   FP32 1200^2       11.8 / 9.7, 15.3 / 12.0     7.9 / 7.6,  8.9 / 8.3
+//        1400 x 1300  14.2 / 11.7, 16.6 / 14.9    7.9 / 8.3,  8.7 / 8.8
+//        1472 x 1424  13.8 / 11.6, 19.3 / 15.5    8.2 / 8.5,  9.1 / 9.0
+//        1449 x 1447  17.9 / 12.2, 27.0 / 18.1   11.4 / 8.5, 13.1 / 8.7
+//   FP64 1024 x 768   17.4 / 9.9,  21.8 / 14.3   13.2 / 7.4, 18.2 / 12.0
+//        1536 x 1200  26.0 / 16.3, 37.9 / 26.7   14.3 / 13.2, 29.4 / 18.4
+// so one young nucleus on 1.7 .. 2 Mi cells of aligned FP32 rows is 3 to 5 %
+// slower without, and everything else faster; past 2 Mi cells chunk lists join
+// in.
 bool status_ok(const kg_solver_s &h)
 {
     return h.cells() > (size_t)1 << 21 &&
