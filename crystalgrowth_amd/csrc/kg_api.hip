@@ -281,8 +281,8 @@ void free_all(kg_solver_s *h)
         (void)hipStreamSynchronize(h->stream);
     kg::free_adjoint(h->adj);
     h->adj = nullptr;
-    void *bufs[] = {h->phi[0], h->phi[1], h->T[0], h->T[1], h->theta_mem, h->temps,
-                    h->partials, h->red, h->disks, h->stat, h->image};
+    void *bufs[] = {h->phi[0], h->phi[1], h->T[0], h->T[1], h->theta, h->temps, h->partials,
+                    h->red, h->disks, h->stat, h->image, h->theta_alt};
     for (void *b : bufs)
         if (b)
             (void)hipFree(b);
@@ -454,34 +454,21 @@ int kg_create(int nx, int ny, int precision, const kg_params *p, kg_handle *out)
         free_all(h);
         return hip_fail(e, "stream/event creation");
     }
-    const size_t field = kg::padded_bytes(h->field_bytes());
-    void **bufs[] = {&h->phi[0], &h->phi[1], &h->T[0], &h->T[1]};
-    bool ok = true;
-    for (void **b : bufs)
-        if (ok && hipMalloc(b, field) != hipSuccess) {
+    void **bufs[] = {&h->phi[0], &h->phi[1], &h->T[0], &h->T[1], &h->theta};
+    for (void **b : bufs) {
+        if (hipMalloc(b, kg::padded_bytes(h->field_bytes())) != hipSuccess) {
             *b = nullptr;
-            ok = false;
-        }
-    // launches of several steps take a second theta, in the same allocation;
-    // without room for it the grid takes single steps
-    if (ok && kg::multi_shape(nx, ny, h->esize()) != 0) {
-        const size_t second = (field + 255) / 256 * 256;
-        if (hipMalloc(&h->theta_mem, second + field) == hipSuccess)
-            h->theta_alt = static_cast<char *>(h->theta_mem) + second;
-        else {
-            h->theta_mem = nullptr;
-            (void)hipGetLastError();
+            free_all(h);
+            return fail(KG_ERR_OUT_OF_MEMORY, "hipMalloc of the fields failed");
         }
     }
-    if (ok && !h->theta_mem && hipMalloc(&h->theta_mem, field) != hipSuccess) {
-        h->theta_mem = nullptr;
-        ok = false;
+    // launches of several steps take a second theta; without room for it the
+    // grid takes single steps
+    if (kg::multi_shape(nx, ny, h->esize()) != 0 &&
+        hipMalloc(&h->theta_alt, kg::padded_bytes(h->field_bytes())) != hipSuccess) {
+        h->theta_alt = nullptr;
+        (void)hipGetLastError();
     }
-    if (!ok) {
-        free_all(h);
-        return fail(KG_ERR_OUT_OF_MEMORY, "hipMalloc of the fields failed");
-    }
-    h->theta = h->theta_mem;
     if (hipMalloc(&h->partials, kg::reduce_partials_size() * sizeof(double)) != hipSuccess ||
         hipMalloc(&h->red, sizeof(kg::ReduceOut)) != hipSuccess) {
         free_all(h);

@@ -45,7 +45,6 @@ struct kg_solver_s {
     void *T[2] = {nullptr, nullptr};
     void *theta = nullptr;
     void *theta_alt = nullptr;  // other theta buffer of launches of several steps (null: none)
-    void *theta_mem = nullptr;  // allocation of both
     void *temps = nullptr;  // 6 fields, two-pass kernel only
     double *partials = nullptr;
     kg::ReduceOut *red = nullptr;
