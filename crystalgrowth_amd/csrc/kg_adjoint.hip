@@ -124,8 +124,9 @@ __device__ __forceinline__ double row_sum(double v)
 // reads phi, T, theta and three adjoints and writes three (36 B in FP32);
 // four kernels through 17 temporary fields moved some 200 B.  us per step:
 // 512^2 FP32 30 -> 7.7, 24 members of 128^2 .. 512^2 (2.6 M cells) 184 -> 27.
-// Bound by VALU work (1.7 pass-1 cells per output cell) and, on small grids,
-// by the chain of four barriers.  Tiles and threads measured on whole
+// Bound by a tile's chain of loads and four barriers (0.19 of the VALU's issue
+// slots at 512^2, 0.53 on the members) and by VALU work (1.7 pass-1 cells per
+// output cell).  Tiles and threads measured on whole
 // adjoints, us (512^2 FP32 / FP64, the 24 members FP32 / FP64, 190 x 133
 // FP64): 32 x 8 on 256 threads 3725 / 5165 / 8380 / 17045 / 1537, on 512
 // 3647 / 5584 / 9353 / 19442 / 1431; 32 x 16 on 256 3960 / 5290 / 7847 /

@@ -25,8 +25,8 @@ struct StepArgs {
     R *phi_out;
     R *T_out;
     R *theta;        // persistent angle, updated in place where a branch fires
-    // small tiles only: old angles in another buffer, all of theta is then
-    // written (nullptr: in theta itself)
+    // old angles in another buffer, all of theta is then written: small tiles
+    // (nullptr: in theta itself) and k_step_batch_direct
     const R *theta_in;
     int nx, ny;
     int boundary;    // 0 periodic, 1 zero-flux

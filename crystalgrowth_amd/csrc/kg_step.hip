@@ -2,8 +2,9 @@
 //
 // One explicit-Euler step = the reference's pass 1 (_computeGradientLaplacian,
 // src/Kobayashi.cpp:125-175) and pass 2 (_evolution, :177-221).  The fused
-// kernel does both in one launch per step (grids of up to 2 Mi cells take small
-// tiles, and up to three steps a launch: k_step_small, k_step_multi):
+// kernel does both in one launch per step (small grids take small tiles, and up to
+// three steps a launch: k_step_small, k_step_multi; small_shape and multi_shape
+// say which grids):
 //   * a 512-thread block owns a 64 x 30 output tile; phi (halo 2) and T
 //     (halo 1) are staged in LDS as rows x0-4 .. x0+67, loaded with aligned
 //     16-byte vector loads whenever nx % 4 == 0 (halo segments beyond an
@@ -1792,7 +1793,8 @@ __device__ __forceinline__ int block_excl_scan(int v, int *wsum, int &total)
 // at position j / 8 of that XCD's sequence, cw * ch entries per chunk
 // (tiles outside the member and the last round's missing chunks are padding
 // entries, member -1).  *count = entries, or -1: no valid answer, or every
-// chunk live (the full table).  *periods counts the lists made.
+// chunk live and none busy (the full table).  *periods counts the lists made that
+// leave chunks out.
 template <typename R>
 __global__ __launch_bounds__(1024) void k_batch_compact(const StepArgs<R> *__restrict__ members,
                                                         const int4 *__restrict__ chunks,

@@ -155,8 +155,8 @@ int kg_get_temperature(kg_handle h, void *dst, size_t bytes);
 int kg_get_angle(kg_handle h, void *dst, size_t bytes);
 /* Replaces the state; theta may be NULL (then 0).  Does not touch the counter. */
 int kg_set_fields(kg_handle h, const void *phi, const void *T, const void *theta, size_t bytes);
-/* Device addresses of the current fields (valid until the next kg_step or
- * kg_reset*) and the handle's stream (hipStream_t). */
+/* Device addresses of the current fields (valid until the next kg_step,
+ * kg_reset* or kg_adjoint) and the handle's stream (hipStream_t). */
 int kg_device_fields(kg_handle h, void **phi, void **T, void **theta);
 int kg_get_stream(kg_handle h, void **stream);
 
