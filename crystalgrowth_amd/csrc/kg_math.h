@@ -48,9 +48,9 @@ __device__ __forceinline__ float kg_atan(float x)
 __device__ __forceinline__ float kg_atan_ratio(float y, float x)
 {
     const float ax = fabsf(x), ay = fabsf(y);
-    const float mx = fmaxf(ax, ay), mn = fminf(ax, ay);
-    float p = atan_unit(mn * fast_rcp(mx));
-    p = ay > ax ? 1.57079637f - p : p;
+    const bool steep = ay > ax;  // (selects, where fminf and fmaxf would drop a NaN)
+    float p = atan_unit((steep ? ax : ay) * fast_rcp(steep ? ay : ax));
+    p = steep ? 1.57079637f - p : p;
     return copysignf(p, __uint_as_float(__float_as_uint(x) ^ __float_as_uint(y)));
 }
 
